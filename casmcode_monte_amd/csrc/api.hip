@@ -421,8 +421,7 @@ struct mcg_handle {
   CanonParams *d_kp = nullptr;
   std::vector<CanonParams> kp;
   int32_t *d_list = nullptr;
-  int canon_lds = 0;       // the largest canon_lds_bytes at creation
-  int canon_walk_lds = 0;  // the kernel's dynamic LDS
+  int canon_lds = 0;  // the largest canon_lds_bytes at creation
   bool canonical() const { return mode == MCG_MODE_CANONICAL; }
   // NFOLD: per-chain parameters (the class arrays share d_list)
   NfoldParams *d_np = nullptr;
@@ -780,7 +779,6 @@ void fill_canonical_params(mcg_handle *h, int c, int64_t nA, CanonParams &P) {
   while (P.mark_mask < 16383 && (int64_t)P.mark_mask + 1 < P.n) P.mark_mask = 2 * P.mark_mask + 1;
   while (P.mark_mask > 2047 && canon_walk_lds_bytes(P) > share) P.mark_mask >>= 1;
   while (P.mark_mask > 255 && canon_walk_lds_bytes(P) > LDS_LIMIT) P.mark_mask >>= 1;
-  h->canon_walk_lds = std::max(h->canon_walk_lds, canon_walk_lds_bytes(P));
   P.negJ = -h->J1;
   P.lat_off = h->lat_off[c];
   const double beta = 1.0 / (h->kb * ch.temperature);  // occupation_metropolis.hh:108-109
@@ -3030,9 +3028,11 @@ int mcg_run(mcg_handle *h, int64_t n_passes) {
     rc = exact_launch(h, n_passes, 0);
     if (rc != MCG_OK) return rc;
   } else if (h->canonical()) {
+    int lds = 0;
+    for (int c = 0; c < h->n_chains; ++c)
+      if (h->active[c]) lds = std::max(lds, canon_walk_lds_bytes(h->kp[c]));
     launch_canonical(h->d_kp, h->d_xs, h->d_lat, h->d_list, h->d_series, h->series_cap,
-                     h->d_active, h->n_chains, n_passes, h->sample_period,
-                     h->canon_walk_lds, h->stream);
+                     h->d_active, h->n_chains, n_passes, h->sample_period, lds, h->stream);
   } else if (h->nfold()) {
     bool general = false;
     for (int c = 0; c < h->n_chains; ++c)
