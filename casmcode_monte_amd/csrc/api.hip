@@ -2187,12 +2187,17 @@ int exact_launch(mcg_handle *h, int64_t n_passes, int64_t n_steps) {
       scratch = std::max(scratch, 4 * (h->xp[c].rows + h->xp[c].cols));
     }
   }
-  if (any_hbm) {
+  // alone, the HBM chains take the handle's stream (the fork and join of a second
+  // one cost 25 us on MI355X: a 1x1 chain, one attempt 46 and 16)
+  const bool fork = any_hbm && any_fit;
+  if (fork) {
     HIP_TRY(hipEventRecord(h->ev_fork, h->stream));
     HIP_TRY(hipStreamWaitEvent(h->stream2, h->ev_fork, 0));
+  }
+  if (any_hbm) {
     launch_exact(h->d_xp, h->d_xs, h->d_lat, h->d_series, h->series_cap, h->d_mask_hbm,
                  h->n_chains, n_passes, n_steps, h->sample_period, scratch, false, false,
-                 h->stream2);
+                 fork ? h->stream2 : h->stream);
     HIP_TRY(hipGetLastError());
   }
   if (any_fit) {
@@ -2201,7 +2206,7 @@ int exact_launch(mcg_handle *h, int64_t n_passes, int64_t n_steps) {
                  !(h->options & MCG_OPT_EXACT_SCALAR_WALK), h->stream);
     HIP_TRY(hipGetLastError());
   }
-  if (any_hbm) {
+  if (fork) {
     HIP_TRY(hipEventRecord(h->ev_join, h->stream2));
     HIP_TRY(hipStreamWaitEvent(h->stream, h->ev_join, 0));
   }
