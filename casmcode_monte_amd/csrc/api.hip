@@ -692,12 +692,13 @@ void fill_exact_params(mcg_handle *h, int c, ExactParams &P) {
 }
 
 // Device masks of the active EXACT chains whose lattice fits the block walk's
-// LDS and of the others (scalar walk on the HBM lattice).
+// LDS and of those that take the scalar walk on the HBM lattice, always or when a
+// launch is short (block_from).
 int exact_update_masks(mcg_handle *h) {
   std::vector<uint8_t> m(2 * (size_t)h->n_chains);
   for (int c = 0; c < h->n_chains; ++c) {
     m[c] = h->active[c] && h->xfit[c];
-    m[h->n_chains + c] = h->active[c] && !h->xfit[c];
+    m[h->n_chains + c] = h->active[c] && (!h->xfit[c] || h->xp[c].block_from > 0);
   }
   HIP_TRY(copy_sync(h, h->d_mask_lds, m.data(), 2 * (size_t)h->n_chains, hipMemcpyHostToDevice));
   return MCG_OK;
@@ -706,14 +707,26 @@ int exact_update_masks(mcg_handle *h) {
 // Set chain c's EXACT path from its parameters: the block walk (or, with
 // MCG_OPT_EXACT_SCALAR_WALK, the scalar walk) in LDS when its lattice fits, else
 // the scalar walk on HBM (fold scratch in LDS).
+//
+// Setting up the classes of a lattice that a byte a site does not fit LDS takes longer
+// than few attempts do on HBM (MI355X: 400x400 sites 300 us, 512x512 480, against 16 and
+// 0.47 an attempt), so it takes the block walk from n / 300 attempts on: where the two
+// meet at both sizes.  Smaller lattices always do: their set-up takes no longer than the
+// copy of their bytes into LDS did.
 int exact_choose_path(mcg_handle *h, int c) {
-  auto const &P = h->xp[c];
+  auto &P = h->xp[c];
   const bool scalar = h->options & MCG_OPT_EXACT_SCALAR_WALK;
   const int64_t lds = scalar ? exact_scalar_lds_bytes(P) : exact_block_lds_bytes(P);
+  const bool scratch_fits = 4 * ((int64_t)P.rows + P.cols) <= EXACT_LDS_MAX;
   h->xlds[c] = (int)lds;
   h->xfit[c] = lds <= (scalar ? EXACT_LDS_MAX : EXACT_BLOCK_LDS_MAX) &&
                (scalar || (P.n > 1 && P.n <= EXACT_BLOCK_MAX_SITES));
-  if (!h->xfit[c] && 4 * ((int64_t)P.rows + P.cols) > EXACT_LDS_MAX)
+  P.block_from = 0;
+  if (!h->xfit[c])
+    P.block_from = std::numeric_limits<int64_t>::max();
+  else if (exact_scalar_lds_bytes(P) > EXACT_LDS_MAX && scratch_fits)
+    P.block_from = P.n / 300;
+  if (!h->xfit[c] && !scratch_fits)
     return fail(MCG_ERR_ARG, "lattice too large for EXACT mode");
   return MCG_OK;
 }
@@ -2171,7 +2184,8 @@ void tune_cache_store(const std::string &key, const mcg_schedule &s) {
 bool valid_chain(mcg_handle *h, int64_t c) { return h && c >= 0 && c < h->n_chains; }
 
 // EXACT launches: the chains whose lattice fits in LDS run the block walk on the
-// handle's stream; the others run the scalar walk on their HBM lattices on the
+// handle's stream (a short launch of a large one aside, block_from); the others run the
+// scalar walk on their HBM lattices on the
 // second stream at the same time (the two sets touch disjoint chains), and
 // the handle's stream waits for them.
 int exact_launch(mcg_handle *h, int64_t n_passes, int64_t n_steps) {
@@ -2179,12 +2193,13 @@ int exact_launch(mcg_handle *h, int64_t n_passes, int64_t n_steps) {
   bool any_fit = false, any_hbm = false;
   for (int c = 0; c < h->n_chains; ++c) {
     if (!h->active[c]) continue;
-    if (h->xfit[c]) {
+    auto const &P = h->xp[c];
+    if (n_passes * (int64_t)P.n + n_steps >= P.block_from) {
       any_fit = true;
       lds = std::max(lds, h->xlds[c]);
     } else {
       any_hbm = true;
-      scratch = std::max(scratch, 4 * (h->xp[c].rows + h->xp[c].cols));
+      scratch = std::max(scratch, 4 * (P.rows + P.cols));
     }
   }
   // alone, the HBM chains take the handle's stream (the fork and join of a second
@@ -2530,7 +2545,7 @@ int mcg_assign_chain(mcg_handle *h, int64_t chain, const mcg_chain_desc *desc) {
       exact_choose_path(h, (int)chain);
       return prc;
     }
-    HIP_TRY(copy_sync(h, h->d_xp + chain, &P, sizeof(P), hipMemcpyHostToDevice));
+    HIP_TRY(copy_sync(h, h->d_xp + chain, &h->xp[chain], sizeof(P), hipMemcpyHostToDevice));
     {
       const int mrc = exact_update_masks(h);
       if (mrc != MCG_OK) return mrc;

@@ -73,6 +73,10 @@ __global__ __launch_bounds__(64) void exact_kernel(const ExactParams *__restrict
   const ExactParams *P = Pp + c;
   ExactState *St = Sp + c;
   const int32_t rows = P->rows, cols = P->cols, n = P->n;
+  // attempts of this launch: n_passes whole passes and n_steps more, from the
+  // chain's position `step` in its current pass
+  const int64_t total = n_passes * (int64_t)n + n_steps;
+  if (!LDS_LATTICE && total >= P->block_from) return;  // exact_block_kernel's
   const uint64_t magic = P->div_magic;
   const uint32_t neg_mask = P->neg_mask, full_mask = P->full_mask;
   const int fold = P->fold;
@@ -103,10 +107,7 @@ __global__ __launch_bounds__(64) void exact_kernel(const ExactParams *__restrict
     return mt_temper(w);
   };
 
-  // attempts of this launch: n_passes whole passes and n_steps more, from the
-  // chain's position `step` in its current pass
   int32_t step = (int32_t)St->step;
-  const int64_t total = n_passes * (int64_t)n + n_steps;
   for (int64_t done = 0; done < total; ++done) {
     {
       // propose: l = uniform_int_distribution<long>(0, n-1) (Lemire)
@@ -325,6 +326,8 @@ __global__ __launch_bounds__(EXACT_THREADS) void exact_block_kernel(const ExactP
   ExactState *St = Sp + c;
   mcg_sample *series = series_pool + (int64_t)c * series_cap;
   const int32_t rows = P->rows, cols = P->cols, n = P->n;
+  const int64_t total = n_passes * (int64_t)n + n_steps;
+  if (total < P->block_from) return;  // exact_kernel's
   const uint64_t magic = P->div_magic;
   const uint32_t neg_mask = P->neg_mask, full_mask = P->full_mask, mmask = P->mark_mask;
   const uint32_t always = neg_mask | full_mask;
@@ -369,7 +372,6 @@ __global__ __launch_bounds__(EXACT_THREADS) void exact_block_kernel(const ExactP
   }
   const int64_t pos0 = St->pos;
   const int32_t step0 = (int32_t)St->step;
-  const int64_t total = n_passes * (int64_t)n + n_steps;
   __syncthreads();
   for (int l = threadIdx.x; l < n; l += EXACT_THREADS) {
     if (g_lat[l] <= 0) continue;

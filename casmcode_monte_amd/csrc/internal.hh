@@ -33,6 +33,7 @@ struct ExactParams {
   double dq[EXACT_NCLASS];  // fl(dE_k / n_unitcells), occupation_metropolis.hh:141
   double negJ;               // -J, for the row/column fold
   int64_t lat_off;           // byte offset of this chain's lattice in the pool
+  int64_t block_from;        // launches of fewer attempts take the scalar walk on HBM
 };
 
 // The block walk's lattice: a site's class in four bits, so at most 2^18 sites

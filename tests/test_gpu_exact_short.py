@@ -1,5 +1,6 @@
-"""EXACT launches of a few attempts: chains of both walks in one launch, a handle whose chains
-all live in HBM.  Bit-exact against the scalar walk (OPT_EXACT_SCALAR_WALK)."""
+"""EXACT launches of a few attempts: chains on either side of the length from which a large
+lattice takes the block walk, chains of both walks in one launch, a handle whose chains all
+live in HBM.  Bit-exact against the scalar walk (OPT_EXACT_SCALAR_WALK)."""
 import numpy as np
 import pytest
 
