@@ -476,6 +476,9 @@ struct mcg_handle {
   uint8_t *d_mask_even = nullptr, *d_mask_ring = nullptr;
   int32_t *d_ring_list = nullptr;
   int n_ring_active = 0, ring_per_chain = 1, ring_lds_bytes = 0;
+  // the words kernel's plans for the active even and ring-coloured chains
+  WordPlan even_words, ring_words;
+  bool words_dirty = true;
   bool any_ring() const { return n_ring_active > 0; }
   bool any_even() const {
     return std::count(active.begin(), active.end(), 1) > n_ring_active;
@@ -1493,6 +1496,7 @@ int checker_update_masks(mcg_handle *h) {
     }
   }
   HIP_TRY(copy_sync(h, h->d_mask_even, m.data(), m.size(), hipMemcpyHostToDevice));
+  h->words_dirty = true;
   h->n_ring_active = (int)ring.size();
   // about four units per thread of a 256-thread block
   h->ring_per_chain = (int)std::min<int64_t>(4096, std::max<int64_t>(1, (max_units + 1023) / 1024));
@@ -3080,10 +3084,15 @@ int mcg_run(mcg_handle *h, int64_t n_passes) {
   } else if (h->checker_lds) {
     // parity-coloured chains on the handle's stream, ring-coloured ones beside
     // them on the second stream (they touch disjoint chains)
+    if (h->words_dirty) {  // (a look at every chain: 4096 of 8x8, one pass 117 and 47 us)
+      h->even_words = plan_words(h, false);
+      h->ring_words = plan_words(h, true);
+      h->words_dirty = false;
+    }
     if (h->any_ring()) {
       HIP_TRY(hipEventRecord(h->ev_fork, h->stream));
       HIP_TRY(hipStreamWaitEvent(h->stream2, h->ev_fork, 0));
-      const WordPlan rw = plan_words(h, true);
+      const WordPlan &rw = h->ring_words;
       if (rw.oct)
         launch_checker_words(h->d_cp, h->d_cs, h->d_lat, h->d_tab, h->d_series, h->series_cap,
                              h->d_mask_ring, h->n_chains, n_passes, h->sample_period, true,
@@ -3094,7 +3103,7 @@ int mcg_run(mcg_handle *h, int64_t n_passes) {
                                 h->checker_lds_bytes, h->checker_block, h->stream2);
       HIP_TRY(hipGetLastError());
     }
-    const WordPlan ew = plan_words(h, false);
+    const WordPlan &ew = h->even_words;
     if (ew.oct)
       launch_checker_words(h->d_cp, h->d_cs, h->d_lat, h->d_tab, h->d_series, h->series_cap,
                            h->d_mask_even, h->n_chains, n_passes, h->sample_period, false,
