@@ -607,6 +607,10 @@ __global__ __launch_bounds__(1024) void checker_words_kernel(
   const bool odd = RING && (L0 & 1);
   const int n_even = (L0 + 1) >> 1, n_odd = L0 >> 1;
   const int hw = (n_even + W - 1) / W, rs = 2 * hw + 1;
+  // the place in its word of the site that a line's first has to its west (a choice between
+  // variables inside the lambda below would put them and the sums into scratch memory: 1024
+  // chains of 31x31, eight passes 156 us, so 105)
+  const int wrap_place = (n_odd + (odd ? 1 : 0) - 1) % W;
   if (RING) {
     for (int i = t; i < 128; i += nt) ltab[i] = tab[((i & 0x78) << 1) | (i & 7)];
   } else if (NNN) {
@@ -644,7 +648,7 @@ __global__ __launch_bounds__(1024) void checker_words_kernel(
     const bool last = w == hw - 1;
     const int wrap_at = odd ? hw - 1 : 2 * hw - 1;
     const int from = a ? (last ? 0 : w + 1) : (w ? hw + w - 1 : wrap_at);
-    const int place = a ? (last ? (n_odd - 1) % W : W - 1) : (w ? W - 1 : ((odd ? n_even : n_odd) - 1) % W);
+    const int place = a ? (last ? (n_odd - 1) % W : W - 1) : (w ? W - 1 : wrap_place);
     const uint32_t enter = a && last && odd ? 0u : 1u;
     auto shifted = [&](const uint32_t *line) __attribute__((always_inline)) {
       const uint32_t x = line[(a ? 0 : hw) + w], y = line[from];
