@@ -1000,6 +1000,24 @@ __global__ __launch_bounds__(BAND_BLOCK) void checker_seam_kernel(
   block_add_deltas(P, dS1, dS2, dM, nacc, red);
 }
 
+// Sum over a wavefront, in lane 63.
+__device__ __forceinline__ int64_t wave_sum64(int64_t v) {
+  auto add = [&](int lo, int hi) __attribute__((always_inline)) {
+    v += (int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
+  };
+#define MCG_DPP(CTRL, ROWS, ZERO)                                              \
+  add(__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, ZERO),           \
+      __builtin_amdgcn_update_dpp(0, (int)(v >> 32), CTRL, ROWS, 0xf, ZERO))
+  MCG_DPP(0x111, 0xf, true);  // row_shr 1, 2, 4, 8
+  MCG_DPP(0x112, 0xf, true);
+  MCG_DPP(0x114, 0xf, true);
+  MCG_DPP(0x118, 0xf, true);
+  MCG_DPP(0x142, 0xa, false);  // row_bcast 15, 31
+  MCG_DPP(0x143, 0xc, false);
+#undef MCG_DPP
+  return v;
+}
+
 // After the last colour of a pass, or of up to CHECKER_AHEAD of them, a workgroup per
 // chain with a wavefront per pass: the slots' sums into the state (and the slots back to
 // zero), the pass counter on, sample records when due.  A launch costs 4.4 us whatever
@@ -1015,13 +1033,13 @@ __global__ __launch_bounds__(64 * CHECKER_AHEAD) void checker_record_kernel(
   int64_t d[4];
 #pragma unroll
   for (int q = 0; q < 4; ++q) d[q] = part[q];
+  CheckerState S = Sp[c];  // (before anything is waited for)
   if (!active[c]) return;
-  CheckerState S = Sp[c];
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     part[q] = 0;
-    for (int o = 32; o > 0; o >>= 1) d[q] += (int64_t)__shfl_xor((long long)d[q], o, 64);
-    if (lane == 0) sum[p][q] = d[q];
+    d[q] = wave_sum64(d[q]);
+    if (lane == 63) sum[p][q] = d[q];
   }
   __syncthreads();
   if (threadIdx.x != 0) return;
