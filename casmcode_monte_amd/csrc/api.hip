@@ -2030,28 +2030,28 @@ int rebuild_work(mcg_handle *h) {
 }
 
 // One pass of the HBM path, `ahead` passes after the last record launch: one launch per
-// colour over the work list, then the pass-counter/sample-record launch (the bit-packed
-// path's only if it is due or `last`).  Returns the passes since the last record.
+// colour over the work list, then the pass-counter/sample-record launch if it is due or
+// `last`.  Returns the passes since the last record.
 int enqueue_pass(mcg_handle *h, int ahead, bool last) {
   if (h->bit.n_items > 0)
     launch_bit_pass(h->d_cp, h->d_cs, h->d_tab, h->bit, ahead, h->stream);
   else if (h->n_bands > 0)
     launch_checker_band(h->d_cp, h->d_cs, h->d_lat, h->d_tab, h->d_band, h->n_bands,
-                        h->band_ring_bytes, h->stream);
+                        h->band_ring_bytes, ahead, h->stream);
   else if (h->n_pairs > 0)
     for (int lc = 0; lc < h->ncolor / 2; ++lc)
       launch_checker_pair(h->d_cp, h->d_cs, h->d_lat, h->d_tab, h->d_pair, h->n_pairs, lc,
-                          h->pair_lds, h->tile_grid, h->stream);
+                          h->pair_lds, h->tile_grid, ahead, h->stream);
   else if (h->n_work > 0)
     for (int color = 0; color < h->ncolor; ++color)
       launch_checker_color(h->d_cp, h->d_cs, h->d_lat, h->d_tab, h->d_work, h->n_work, color,
-                           h->units_per_thread, h->stream);
+                           h->units_per_thread, ahead, h->stream);
   if (h->any_ring())
     launch_checker_ring_pass(h->d_cp, h->d_cs, h->d_lat, h->d_tab, h->d_ring_list,
                              h->n_ring_active, h->ring_per_chain,
-                             h->lattice == MCG_LATTICE_SC ? 3 : 2, h->stream);
+                             h->lattice == MCG_LATTICE_SC ? 3 : 2, ahead, h->stream);
   ++ahead;
-  if (h->bit.n_items > 0 && !h->any_ring() && !last && ahead < CHECKER_AHEAD) return ahead;
+  if (!last && ahead < CHECKER_AHEAD) return ahead;
   launch_checker_record(h->d_cs, h->d_parts, h->d_series, h->series_cap, h->d_active, h->n_chains,
                         h->sample_period, ahead, h->stream);
   return 0;

@@ -508,7 +508,7 @@ template <int UPT>
 __global__ __launch_bounds__(HBM_BLOCK) void checker_color_kernel(
     const CheckerParams *__restrict__ Pp, CheckerState *__restrict__ Sp,
     int8_t *__restrict__ lat_pool, const uint32_t *__restrict__ tables,
-    const int32_t *__restrict__ work, int color) {
+    const int32_t *__restrict__ work, int color, int ahead) {
   constexpr int BLOCKS_PER_ITEM = MAX_UNITS_PER_THREAD / UPT;
   __shared__ int red[4][HBM_BLOCK / 64];
   const int item = blockIdx.x / BLOCKS_PER_ITEM;
@@ -516,11 +516,11 @@ __global__ __launch_bounds__(HBM_BLOCK) void checker_color_kernel(
   const int c = work[2 * item];
   const int64_t u0 =
       (int64_t)work[2 * item + 1] * UNITS_PER_ITEM + (int64_t)sub * HBM_BLOCK * UPT;
-  const CheckerParams P = Pp[c];
+  const CheckerParams P = checker_ahead(Pp, c, ahead);
   CheckerState *St = Sp + c;
   const LineGeom g = line_geom(P);
   const int64_t nu = n_units(g);
-  const int64_t pass = St->n_pass;
+  const int64_t pass = St->n_pass + ahead;
   const uint32_t *tab = tables + P.tab_off;
   uint8_t *lat = reinterpret_cast<uint8_t *>(lat_pool + P.lat_off);
   int dS1 = 0, dS2 = 0, dM = 0, nacc = 0;
@@ -580,14 +580,14 @@ __device__ __forceinline__ int xcd_item(int i, int n) {
 __global__ __launch_bounds__(PAIR_BLOCK) void checker_pair_kernel(
     const CheckerParams *__restrict__ Pp, CheckerState *__restrict__ Sp,
     int8_t *__restrict__ lat_pool, const uint32_t *__restrict__ tables,
-    const int32_t *__restrict__ work, int line_class) {
+    const int32_t *__restrict__ work, int line_class, int ahead) {
   __shared__ int red[4][PAIR_BLOCK / 64];
   const int32_t *item = work + 4 * xcd_item(blockIdx.x, gridDim.x);
   const int c = item[0];
-  const CheckerParams P = Pp[c];
+  const CheckerParams P = checker_ahead(Pp, c, ahead);
   CheckerState *St = Sp + c;
   const LineGeom g = line_geom(P);
-  const int64_t pass = St->n_pass;
+  const int64_t pass = St->n_pass + ahead;
   const uint32_t *tab = tables + P.tab_off;
   uint8_t *lat = reinterpret_cast<uint8_t *>(lat_pool + P.lat_off);
   const int upl = chunk_path(g) ? (g.half >> 4) : g.qpl;  // units per half line
@@ -672,7 +672,7 @@ __device__ __forceinline__ TileGeom tile_geom(const CheckerParams *__restrict__ 
 __global__ __launch_bounds__(PAIR_BLOCK) void checker_tile_kernel(
     const CheckerParams *__restrict__ Pp, CheckerState *__restrict__ Sp,
     int8_t *__restrict__ lat_pool, const uint32_t *__restrict__ tables,
-    const int32_t *__restrict__ work, int n_items, int line_class) {
+    const int32_t *__restrict__ work, int n_items, int line_class, int ahead) {
   extern __shared__ __align__(16) uint8_t region[];
   __shared__ int red[4][PAIR_BLOCK / 64];
   __shared__ uint32_t tab[CHECKER_NTAB];  // acceptance table of the current tile's chain
@@ -727,10 +727,10 @@ __global__ __launch_bounds__(PAIR_BLOCK) void checker_tile_kernel(
     const int nxt = it + (int)gridDim.x;
     if (nxt < n_items) MCG_TILE_FETCH(nxt);  // in flight while this tile is updated
     const TileGeom t = tile_geom(Pp, work, it);
-    const CheckerParams P = Pp[t.c];
+    const CheckerParams P = checker_ahead(Pp, t.c, ahead);
     CheckerState *St = Sp + t.c;
     const LineGeom g = line_geom(P);
-    const int64_t pass = St->n_pass;
+    const int64_t pass = St->n_pass + ahead;
     uint8_t *lat = reinterpret_cast<uint8_t *>(lat_pool + P.lat_off);
     const int upl = g.half >> 4;
     const bool d3 = P.ndim == 3;
@@ -901,14 +901,14 @@ __device__ __forceinline__ void block_add_deltas(const CheckerParams &P, int dS1
 __global__ __launch_bounds__(BAND_BLOCK) void checker_band_kernel(
     const CheckerParams *__restrict__ Pp, CheckerState *__restrict__ Sp,
     int8_t *__restrict__ lat_pool, const uint32_t *__restrict__ tables,
-    const int32_t *__restrict__ work) {
+    const int32_t *__restrict__ work, int ahead) {
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ uint32_t tab[CHECKER_NTAB];
   __shared__ int red[4][BAND_BLOCK / 64];
   const int c = work[3 * blockIdx.x], j0 = work[3 * blockIdx.x + 1], H = work[3 * blockIdx.x + 2];
-  const CheckerParams P = Pp[c];
+  const CheckerParams P = checker_ahead(Pp, c, ahead);
   CheckerState *St = Sp + c;
-  const int64_t pass = St->n_pass;
+  const int64_t pass = St->n_pass + ahead;
   for (int i = threadIdx.x; i < CHECKER_NTAB; i += BAND_BLOCK) tab[i] = tables[P.tab_off + i];
   uint8_t *lat = reinterpret_cast<uint8_t *>(lat_pool + P.lat_off);
   BandCtx b;
@@ -971,12 +971,12 @@ __global__ __launch_bounds__(BAND_BLOCK) void checker_band_kernel(
 __global__ __launch_bounds__(BAND_BLOCK) void checker_seam_kernel(
     const CheckerParams *__restrict__ Pp, CheckerState *__restrict__ Sp,
     int8_t *__restrict__ lat_pool, const uint32_t *__restrict__ tables,
-    const int32_t *__restrict__ work) {
+    const int32_t *__restrict__ work, int ahead) {
   __shared__ int red[4][BAND_BLOCK / 64];
   const int c = work[3 * blockIdx.x], j0 = work[3 * blockIdx.x + 1], H = work[3 * blockIdx.x + 2];
-  const CheckerParams P = Pp[c];
+  const CheckerParams P = checker_ahead(Pp, c, ahead);
   CheckerState *St = Sp + c;
-  const int64_t pass = St->n_pass;
+  const int64_t pass = St->n_pass + ahead;
   const uint32_t *tab = tables + P.tab_off;
   uint8_t *lat = reinterpret_cast<uint8_t *>(lat_pool + P.lat_off);
   const LineGeom g = line_geom(P);
@@ -1021,8 +1021,9 @@ __device__ __forceinline__ int64_t wave_sum64(int64_t v) {
 // After the last colour of a pass, or of up to CHECKER_AHEAD of them, a workgroup per
 // chain with a wavefront per pass: the slots' sums into the state (and the slots back to
 // zero), the pass counter on, sample records when due.  A launch costs 4.4 us whatever
-// it does (MI355X), so the bit-packed path makes one for eight passes: two lattices of
-// 4096x4096 27 -> 24.8 us a pass, two of 256^3 38.5 -> 35.5, one of 512x512 13.5 -> 11.3.
+// it does (MI355X), so eight passes share one: on bits, two lattices of 4096x4096 27 ->
+// 24.8 us a pass, two of 256^3 38.5 -> 35.5, one of 512x512 13.5 -> 11.3; on bytes, one of
+// 8192x64 31 -> 28.2, 16 of 500x500 55 -> 53.3, 16 of 363x363 (ring) 68 -> 63.4.
 __global__ __launch_bounds__(64 * CHECKER_AHEAD) void checker_record_kernel(
     CheckerState *__restrict__ Sp, int64_t *__restrict__ parts, mcg_sample *__restrict__ series,
     int64_t series_cap, const uint8_t *__restrict__ active, int64_t sample_period) {
@@ -1068,16 +1069,16 @@ static_assert(CHECKER_PARTS == 64, "a lane per slot");
 
 void launch_checker_color(const CheckerParams *P, CheckerState *St, int8_t *lat_pool,
                           const uint32_t *tables, const int32_t *work, int n_work_items,
-                          int color, int upt, hipStream_t stream) {
+                          int color, int upt, int ahead, hipStream_t stream) {
   if (upt == 1)
     hipLaunchKernelGGL(checker_color_kernel<1>, dim3(n_work_items * 4), dim3(HBM_BLOCK), 0,
-                       stream, P, St, lat_pool, tables, work, color);
+                       stream, P, St, lat_pool, tables, work, color, ahead);
   else if (upt == 2)
     hipLaunchKernelGGL(checker_color_kernel<2>, dim3(n_work_items * 2), dim3(HBM_BLOCK), 0,
-                       stream, P, St, lat_pool, tables, work, color);
+                       stream, P, St, lat_pool, tables, work, color, ahead);
   else
     hipLaunchKernelGGL(checker_color_kernel<4>, dim3(n_work_items), dim3(HBM_BLOCK), 0, stream,
-                       P, St, lat_pool, tables, work, color);
+                       P, St, lat_pool, tables, work, color, ahead);
 }
 
 void launch_checker_record(CheckerState *St, int64_t *parts, mcg_sample *series,
@@ -1130,7 +1131,7 @@ hipError_t checker_graph_add_passes(hipGraph_t g, const CheckerParams *P, Checke
       }
     } else if (n_bands > 0) {
       void *args[] = {(void *)&P, (void *)&St, (void *)&lat_pool, (void *)&tables,
-                      (void *)&band_work};
+                      (void *)&band_work, (void *)&ahead};
       hipError_t e = add(reinterpret_cast<void *>(&checker_band_kernel), dim3(n_bands),
                          dim3(BAND_BLOCK), args, (unsigned)ring_bytes);
       if (e == hipSuccess)
@@ -1143,12 +1144,12 @@ hipError_t checker_graph_add_passes(hipGraph_t g, const CheckerParams *P, Checke
         if (pair_lds > 0) {
           void *args[] = {(void *)&P,         (void *)&St,      (void *)&lat_pool,
                           (void *)&tables,    (void *)&pair_work, (void *)&n_pairs,
-                          (void *)&lc};
+                          (void *)&lc,        (void *)&ahead};
           e = add(reinterpret_cast<void *>(&checker_tile_kernel), dim3(tile_grid),
                   dim3(PAIR_BLOCK), args, (unsigned)pair_lds);
         } else {
           void *args[] = {(void *)&P, (void *)&St, (void *)&lat_pool, (void *)&tables,
-                          (void *)&pair_work, (void *)&lc};
+                          (void *)&pair_work, (void *)&lc, (void *)&ahead};
           e = add(reinterpret_cast<void *>(&checker_pair_kernel), dim3(n_pairs),
                   dim3(PAIR_BLOCK), args);
         }
@@ -1157,12 +1158,12 @@ hipError_t checker_graph_add_passes(hipGraph_t g, const CheckerParams *P, Checke
     } else if (n_work_items > 0)
       for (int color = 0; color < ncolor; ++color) {
         void *args[] = {(void *)&P, (void *)&St, (void *)&lat_pool, (void *)&tables,
-                        (void *)&work, (void *)&color};
+                        (void *)&work, (void *)&color, (void *)&ahead};
         hipError_t e = add(color_fn, dim3(color_grid), dim3(HBM_BLOCK), args);
         if (e != hipSuccess) return e;
       }
     ++ahead;
-    if (bit.n_items > 0 && ahead < CHECKER_AHEAD && p + 1 < passes) continue;
+    if (ahead < CHECKER_AHEAD && p + 1 < passes) continue;
     void *args[] = {(void *)&St,         (void *)&parts,  (void *)&series,
                     (void *)&series_cap, (void *)&active, (void *)&sample_period};
     hipError_t e = add(reinterpret_cast<void *>(&checker_record_kernel), dim3(n_chains),
@@ -1175,11 +1176,11 @@ hipError_t checker_graph_add_passes(hipGraph_t g, const CheckerParams *P, Checke
 
 void launch_checker_band(const CheckerParams *P, CheckerState *St, int8_t *lat_pool,
                          const uint32_t *tables, const int32_t *band_work, int n_bands,
-                         int ring_bytes, hipStream_t stream) {
+                         int ring_bytes, int ahead, hipStream_t stream) {
   hipLaunchKernelGGL(checker_band_kernel, dim3(n_bands), dim3(BAND_BLOCK), ring_bytes, stream,
-                     P, St, lat_pool, tables, band_work);
+                     P, St, lat_pool, tables, band_work, ahead);
   hipLaunchKernelGGL(checker_seam_kernel, dim3(n_bands), dim3(BAND_BLOCK), 0, stream, P, St,
-                     lat_pool, tables, band_work);
+                     lat_pool, tables, band_work, ahead);
 }
 
 // ---------------------------------------------------------------------------
@@ -1244,13 +1245,13 @@ void launch_clear_samples(ExactState *xs, CheckerState *cs, int n_chains, hipStr
 
 void launch_checker_pair(const CheckerParams *P, CheckerState *St, int8_t *lat_pool,
                          const uint32_t *tables, const int32_t *pair_work, int n_items,
-                         int line_class, int lds_bytes, int tile_grid, hipStream_t stream) {
+                         int line_class, int lds_bytes, int tile_grid, int ahead, hipStream_t stream) {
   if (lds_bytes > 0)
     hipLaunchKernelGGL(checker_tile_kernel, dim3(tile_grid), dim3(PAIR_BLOCK), lds_bytes, stream,
-                       P, St, lat_pool, tables, pair_work, n_items, line_class);
+                       P, St, lat_pool, tables, pair_work, n_items, line_class, ahead);
   else
     hipLaunchKernelGGL(checker_pair_kernel, dim3(n_items), dim3(PAIR_BLOCK), 0, stream, P, St,
-                       lat_pool, tables, pair_work, line_class);
+                       lat_pool, tables, pair_work, line_class, ahead);
 }
 
 hipError_t checker_pair_set_max_lds(int bytes) {

@@ -35,14 +35,6 @@ __device__ __forceinline__ BitLattice bit_lattice(const CheckerParams &P) {
   return G;
 }
 
-// A chain's parameters in a launch `ahead` passes ahead of the state's counter: its
-// changes go to that pass's slots.
-__device__ __forceinline__ CheckerParams bit_params(const CheckerParams *Pp, int chain, int ahead) {
-  CheckerParams P = Pp[chain];
-  P.parts += ahead * CHECKER_PASS_PARTS;
-  return P;
-}
-
 // Word wi of chain P's lattice (line-major: line, half, word): its first site's
 // byte, and whether it has 32 sites or 16.
 __device__ __forceinline__ int64_t word_byte(const BitLattice &G, int64_t wi, bool &full) {
@@ -174,7 +166,7 @@ __global__ __launch_bounds__(STREAM_BLOCK) void checker_stream_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wi = blockIdx.x * (STREAM_BLOCK / 64) + wave;
   const BitItem it = items[wi];  // (a workgroup's are one chain's; the last may be empty)
-  const CheckerParams P = bit_params(Pp, it.chain, ahead);
+  const CheckerParams P = checker_ahead(Pp, it.chain, ahead);
   const int64_t pass = Sp[it.chain].n_pass + ahead;
   const uint32_t *tab = tables + P.tab_off;
   if (FOUR)
@@ -424,7 +416,7 @@ __global__ __launch_bounds__(512) void checker_plane_kernel(
   extern __shared__ __align__(16) uint32_t planes[];
   __shared__ uint16_t thi[CHECKER_NTAB];
   const BitItem it = items[blockIdx.x];
-  const CheckerParams P = bit_params(Pp, it.chain, ahead);
+  const CheckerParams P = checker_ahead(Pp, it.chain, ahead);
   const int64_t pass = Sp[it.chain].n_pass + ahead;
   const uint32_t *tab = tables + P.tab_off;
   const int t = threadIdx.x, nt = blockDim.x;
@@ -506,7 +498,7 @@ __global__ __launch_bounds__(CUBE_BLOCK) void checker_cube_kernel(
   constexpr bool PAIRS = OCT == 4;
   __shared__ uint32_t thi[PAIRS ? 256 : 64];
   const BitItem it = items[blockIdx.x];
-  const CheckerParams P = bit_params(Pp, it.chain, ahead);
+  const CheckerParams P = checker_ahead(Pp, it.chain, ahead);
   const int64_t pass = Sp[it.chain].n_pass + ahead;
   const uint32_t *tab = tables + P.tab_off;
   const int t = threadIdx.x;

@@ -210,14 +210,14 @@ constexpr int RING_BLOCK = 256;
 __global__ __launch_bounds__(RING_BLOCK) void checker_ring_class_kernel(
     const CheckerParams *__restrict__ Pp, CheckerState *__restrict__ Sp,
     int8_t *__restrict__ lat_pool, const uint32_t *__restrict__ tables,
-    const int32_t *__restrict__ chains, int per_chain, int col) {
+    const int32_t *__restrict__ chains, int per_chain, int col, int ahead) {
   __shared__ int red[4][RING_BLOCK / 64];
   const int c = chains[blockIdx.x / per_chain];
   const int sub = blockIdx.x % per_chain;
-  const CheckerParams P = Pp[c];
+  const CheckerParams P = checker_ahead(Pp, c, ahead);
   CheckerState *St = Sp + c;
   const RingClass k = ring_class(P, col);
-  const int64_t pass = St->n_pass;
+  const int64_t pass = St->n_pass + ahead;
   const uint32_t *tab = tables + P.tab_off;
   uint8_t *lat = reinterpret_cast<uint8_t *>(lat_pool + P.lat_off);
   int dS1 = 0, dS2 = 0, dM = 0, nacc = 0;
@@ -262,11 +262,11 @@ void launch_checker_ring_lds(const CheckerParams *P, CheckerState *St, int8_t *l
 
 void launch_checker_ring_pass(const CheckerParams *P, CheckerState *St, int8_t *lat_pool,
                               const uint32_t *tables, const int32_t *chains, int n_ring,
-                              int per_chain, int ndim, hipStream_t stream) {
+                              int per_chain, int ndim, int ahead, hipStream_t stream) {
   const int ncls = ndim == 3 ? 27 : 9;
   for (int col = 0; col < ncls; ++col)
     hipLaunchKernelGGL(checker_ring_class_kernel, dim3(n_ring * per_chain), dim3(RING_BLOCK), 0,
-                       stream, P, St, lat_pool, tables, chains, per_chain, col);
+                       stream, P, St, lat_pool, tables, chains, per_chain, col, ahead);
 }
 
 hipError_t checker_ring_set_max_lds(int bytes) {

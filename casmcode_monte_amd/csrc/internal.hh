@@ -314,8 +314,8 @@ struct CheckerParams {
 constexpr int CHECKER_PARTS = 64;
 constexpr int CHECKER_PART_STRIDE = 8;  // int64 per slot
 constexpr int CHECKER_PASS_PARTS = CHECKER_PARTS * CHECKER_PART_STRIDE;
-// Passes of the bit-packed path between two record launches at most: its launches are
-// told how far ahead of the state's pass counter they are.
+// Passes between two record launches at most: the launches are told how far ahead of the
+// state's pass counter they are.
 constexpr int CHECKER_AHEAD = 8;
 
 // Acceptance table of a chain: entry (b << 7) | (c1 << 4) | c2 for old spin
@@ -333,6 +333,15 @@ struct CheckerState {
   int64_t n_samples;
   int64_t S3, T3;          // FCC: P3 and the triangle count
 };
+
+// A chain's parameters in a launch `ahead` passes ahead of the state's counter: its
+// changes go to that pass's slots.
+__device__ __forceinline__ CheckerParams checker_ahead(const CheckerParams *Pp, int chain,
+                                                       int ahead) {
+  CheckerParams P = Pp[chain];
+  P.parts += ahead * CHECKER_PASS_PARTS;
+  return P;
+}
 
 // A workgroup's observable changes into its slot of the chain's (by one thread).
 __device__ __forceinline__ void checker_add_part(const CheckerParams &P, int index, long long a1,
@@ -352,7 +361,7 @@ void launch_checker_lds(const CheckerParams *P, CheckerState *St, int8_t *lat_po
 
 void launch_checker_color(const CheckerParams *P, CheckerState *St, int8_t *lat_pool,
                           const uint32_t *tables, const int32_t *work, int n_work_items,
-                          int color, int upt, hipStream_t stream);
+                          int color, int upt, int ahead, hipStream_t stream);
 
 // Chains with an odd edge (checker_ring.hip): ring colourings, natural layout.
 void launch_checker_ring_lds(const CheckerParams *P, CheckerState *St, int8_t *lat_pool,
@@ -364,7 +373,7 @@ void launch_checker_ring_lds(const CheckerParams *P, CheckerState *St, int8_t *l
 // the record follow in launch_checker_record)
 void launch_checker_ring_pass(const CheckerParams *P, CheckerState *St, int8_t *lat_pool,
                               const uint32_t *tables, const int32_t *chains, int n_ring,
-                              int per_chain, int ndim, hipStream_t stream);
+                              int per_chain, int ndim, int ahead, hipStream_t stream);
 hipError_t checker_ring_set_max_lds(int bytes);
 
 // Spins (+1/-1, site order) of sites [first, first + count) of one lattice into
@@ -458,7 +467,7 @@ hipError_t checker_graph_add_passes(hipGraph_t g, const CheckerParams *P, Checke
 // most checker_tile_max_bytes()), tile_grid persistent workgroups.
 void launch_checker_pair(const CheckerParams *P, CheckerState *St, int8_t *lat_pool,
                          const uint32_t *tables, const int32_t *pair_work, int n_items,
-                         int line_class, int lds_bytes, int tile_grid, hipStream_t stream);
+                         int line_class, int lds_bytes, int tile_grid, int ahead, hipStream_t stream);
 hipError_t checker_pair_set_max_lds(int bytes);
 int checker_pair_block();
 int checker_tile_max_bytes();
@@ -467,7 +476,7 @@ int checker_tile_max_bytes();
 // band-edge launch; ring_bytes = checker_band_ring_lines() * L0 (largest chain).
 void launch_checker_band(const CheckerParams *P, CheckerState *St, int8_t *lat_pool,
                          const uint32_t *tables, const int32_t *band_work, int n_bands,
-                         int ring_bytes, hipStream_t stream);
+                         int ring_bytes, int ahead, hipStream_t stream);
 int checker_band_ring_lines();
 hipError_t checker_band_set_max_lds(int bytes);
 
