@@ -48,7 +48,7 @@ constexpr int64_t LDS_LIMIT = 160 * 1024;     // gfx950 LDS per workgroup
 constexpr int64_t EXACT_LDS_MAX = 144 * 1024;  // a sequential chain's dynamic LDS (+ ~10 KB static)
 constexpr int64_t EXACT_BLOCK_LDS_MAX = 156 * 1024;  // the EXACT block walk's, nothing static
 constexpr int64_t CHECKER_LDS_MAX = 128 * 1024;
-constexpr int64_t FCC_LDS_MAX = 140 * 1024;  // lattice; tables, lists and schedule take 19.2 KB static
+constexpr int64_t FCC_LDS_MAX = 140 * 1024;  // lattice; tables, lists and schedule: at most 20 KB static
 // dynamic LDS above half a CU's 160 KB: a workgroup then has its CU to itself
 constexpr int FCC_ONE_PER_CU_LDS = 81 * 1024;
 

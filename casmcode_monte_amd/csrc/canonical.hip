@@ -429,8 +429,7 @@ void launch_canonical(const CanonParams *P, ExactState *S, int8_t *lat_pool, int
 }
 
 hipError_t canonical_set_max_lds(int bytes) {
-  return hipFuncSetAttribute(reinterpret_cast<const void *>(canonical_kernel),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  return set_dynamic_lds(reinterpret_cast<const void *>(canonical_kernel), bytes, true);
 }
 
 }  // namespace mcg

@@ -640,8 +640,8 @@ void launch_exact(const ExactParams *P, ExactState *S, int8_t *lat_pool, mcg_sam
 // block_bytes, scalar_bytes: the most dynamic LDS a block walk and a scalar walk
 // ask for.
 hipError_t exact_set_max_lds(int block_bytes, int scalar_bytes) {
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(exact_block_kernel),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, block_bytes);
+  hipError_t e =
+      set_dynamic_lds(reinterpret_cast<const void *>(exact_block_kernel), block_bytes, true);
   if (e != hipSuccess) return e;
   e = hipFuncSetAttribute(reinterpret_cast<const void *>(exact_kernel<true>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, scalar_bytes);

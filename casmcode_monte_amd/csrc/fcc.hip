@@ -1141,17 +1141,15 @@ void launch_fcc(const CheckerParams *P, CheckerState *St, int8_t *lat_pool, cons
 }
 
 hipError_t fcc_set_max_lds(int bytes) {
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(fcc_bits_kernel<false>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  if (e != hipSuccess) return e;
-  e = hipFuncSetAttribute(reinterpret_cast<const void *>(fcc_lines_kernel),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  if (e != hipSuccess) return e;
-  e = hipFuncSetAttribute(reinterpret_cast<const void *>(fcc_bits_kernel<true>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  if (e != hipSuccess) return e;
-  return hipFuncSetAttribute(reinterpret_cast<const void *>(fcc_kernel<true>),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  const void *fns[] = {reinterpret_cast<const void *>(fcc_bits_kernel<false>),
+                       reinterpret_cast<const void *>(fcc_lines_kernel),
+                       reinterpret_cast<const void *>(fcc_bits_kernel<true>),
+                       reinterpret_cast<const void *>(fcc_kernel<true>)};
+  for (const void *fn : fns) {
+    const hipError_t e = set_dynamic_lds(fn, bytes, false);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 }  // namespace mcg

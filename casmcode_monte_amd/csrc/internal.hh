@@ -51,6 +51,18 @@ inline int64_t exact_scalar_lds_bytes(const ExactParams &P) {
   return (((int64_t)P.n + 15) & ~int64_t(15)) + 4 * ((int64_t)P.rows + P.cols);
 }
 
+// The most dynamic LDS that launches of kernel fn ask for; refused if it does not fit a
+// workgroup's 160 KB beside what fn has static, which is nothing if fn takes its dynamic
+// array to start at LDS address 0 (walk.hh).
+inline hipError_t set_dynamic_lds(const void *fn, int bytes, bool at_zero) {
+  hipFuncAttributes a;
+  const hipError_t e = hipFuncGetAttributes(&a, fn);
+  if (e != hipSuccess) return e;
+  if (a.sharedSizeBytes > (at_zero ? size_t(0) : size_t(160 * 1024 - bytes)))
+    return hipErrorInvalidDeviceFunction;
+  return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+}
+
 // Read-write per-chain state (EXACT, CANONICAL and NFOLD).
 struct ExactState {
   uint64_t mt[MT_N];  // std::mt19937_64 state words

@@ -1126,9 +1126,8 @@ hipError_t kmc_set_max_lds(int general_bytes, int walk_bytes) {
                                            hipFuncAttributeMaxDynamicSharedMemorySize,
                                            general_bytes);
   return e != hipSuccess ? e
-                         : hipFuncSetAttribute(reinterpret_cast<const void *>(kmc_walk_kernel),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               walk_bytes);
+                         : set_dynamic_lds(reinterpret_cast<const void *>(kmc_walk_kernel),
+                                           walk_bytes, true);
 }
 
 }  // namespace mcg

@@ -908,8 +908,7 @@ hipError_t occupant_set_max_lds(int general_bytes, int sgc_bytes) {
                        reinterpret_cast<const void *>(occupant_sgc_kernel<2>),
                        reinterpret_cast<const void *>(occupant_sgc_kernel<3>)};
   for (const void *f : sgc)
-    if (e == hipSuccess)
-      e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, sgc_bytes);
+    if (e == hipSuccess) e = set_dynamic_lds(f, sgc_bytes, true);
   return e;
 }
 

@@ -155,8 +155,9 @@ struct MtRing3 {
 };
 
 // ---- LDS addressed by byte -------------------------------------------------------
-// Kernels whose only LDS is one dynamic array (it starts at address 0) compute
-// byte addresses themselves: the offsets of their fixed parts become immediates.
+// Kernels whose only LDS is one dynamic array (it starts at address 0; set_dynamic_lds
+// refuses one with static LDS) compute byte addresses themselves: the offsets of their
+// fixed parts become immediates.
 using lds_u32 = __attribute__((address_space(3))) uint32_t;
 __device__ __forceinline__ lds_u32 *lds_at(uint32_t byte) { return (lds_u32 *)(uintptr_t)byte; }
 __device__ __forceinline__ void lds_add(uint32_t byte, uint32_t v) {
