@@ -2117,6 +2117,20 @@ WordPlan plan_words(mcg_handle *h, bool ring) {
   return best;
 }
 
+void plan_words_if_changed(mcg_handle *h) {
+  if (!h->words_dirty) return;  // (a look at every chain: 4096 of 8x8, one pass 117 and 47 us)
+  h->even_words = plan_words(h, false);
+  h->ring_words = plan_words(h, true);
+  h->words_dirty = false;
+}
+
+// Every active chain is the words kernel's.
+bool all_on_words(mcg_handle *h) {
+  if (!h->checker_lds || h->fcc()) return false;
+  plan_words_if_changed(h);
+  return (!h->any_even() || h->even_words.oct) && (!h->any_ring() || h->ring_words.oct);
+}
+
 // Autotuner cache key: path (LDS-resident or HBM), lattice, colouring and
 // the size class (log2 of the sites per chain and of the chain count).
 std::string tune_key(const mcg_handle *h) {
@@ -3084,11 +3098,7 @@ int mcg_run(mcg_handle *h, int64_t n_passes) {
   } else if (h->checker_lds) {
     // parity-coloured chains on the handle's stream, ring-coloured ones beside
     // them on the second stream (they touch disjoint chains)
-    if (h->words_dirty) {  // (a look at every chain: 4096 of 8x8, one pass 117 and 47 us)
-      h->even_words = plan_words(h, false);
-      h->ring_words = plan_words(h, true);
-      h->words_dirty = false;
-    }
+    plan_words_if_changed(h);
     if (h->any_ring()) {
       HIP_TRY(hipEventRecord(h->ev_fork, h->stream));
       HIP_TRY(hipStreamWaitEvent(h->stream2, h->ev_fork, 0));
@@ -3604,6 +3614,9 @@ int mcg_autotune(mcg_handle *h, int64_t trial_passes, mcg_schedule *chosen) {
         cands.push_back({b, h->units_per_thread, 1, 0.0, h->band_lines, 0});
       for (int64_t b : {256, 512, 1024})
         cands.push_back({b, h->units_per_thread, 1, 0.0, h->band_lines, 1});
+    } else if (all_on_words(h)) {  // (nothing to choose: the words kernel has its own plan)
+      cands.push_back({h->checker_block, h->units_per_thread, 1, 0.0, h->band_lines,
+                       h->line_tiles});
     } else if (h->checker_lds || h->fcc()) {
       for (int64_t b : {256, 512, 1024})
         if (!(h->fcc_wide && b > 512))
@@ -3615,13 +3628,13 @@ int mcg_autotune(mcg_handle *h, int64_t trial_passes, mcg_schedule *chosen) {
         for (int64_t u : {1, 2, 4})
           for (int64_t g : {1, 8}) cands.push_back({h->checker_block, u, g, 0.0, 0, lt});
       }
+      // in bands, or on bits: lines from the sizes, or a number of them
+      for (int64_t g : {1, 8})
+        cands.push_back({h->checker_block, h->units_per_thread, g, 0.0, -1, 0});
       if (h->lattice == MCG_LATTICE_SQUARE)
         for (int64_t bl : {4, 8, 16, 32})
           for (int64_t g : {1, 8})
             cands.push_back({h->checker_block, h->units_per_thread, g, 0.0, bl, 0});
-      if (h->lattice == MCG_LATTICE_SC)  // on bits
-        for (int64_t g : {1, 8})
-          cands.push_back({h->checker_block, h->units_per_thread, g, 0.0, -1, 0});
     }
     double best_ms = 1e300;
     int rc = MCG_OK;
@@ -3642,6 +3655,7 @@ int mcg_autotune(mcg_handle *h, int64_t trial_passes, mcg_schedule *chosen) {
     if (rc != MCG_OK) return rc;
     tune_cache_store(key, best);
   }
+  if (all_on_words(h)) best.lds_block = h->checker_block;  // (another handle's, if saved)
   int rc = mcg_set_schedule(h, &best);
   if (rc != MCG_OK) return rc;
   h->tuned_ms = best.trial_ms;

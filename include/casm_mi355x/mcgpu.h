@@ -512,8 +512,9 @@ int mcg_check_batch(mcg_handle *h, int64_t n, const int64_t *chains, int64_t obs
  * tune: one wavefront per chain).  Every schedule produces the same
  * trajectories; only the speed changes. */
 typedef struct mcg_schedule {
-  int64_t lds_block;        /* LDS-resident and FCC kernels: threads per workgroup
-                               (256, 512, 1024)                                         */
+  int64_t lds_block;        /* FCC and LDS-resident kernels on bytes: threads per workgroup
+                               (256, 512, 1024).  2D Ising chains in LDS run on bits and
+                               take theirs from their sizes                             */
   int64_t units_per_thread; /* HBM kernels: work units per thread and colour (1, 2, 4)    */
   int64_t graph_passes;     /* HBM path: passes captured per hipGraph replay (1 = none)   */
   double trial_ms;          /* mcg_autotune: time of the chosen schedule on its trial     */
