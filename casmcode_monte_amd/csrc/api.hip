@@ -2124,16 +2124,24 @@ void plan_words_if_changed(mcg_handle *h) {
   h->words_dirty = false;
 }
 
-// Every active chain is the words kernel's.
+// Every active chain is the words kernel's; every active parity-coloured one the
+// bit-packed path's.
 bool all_on_words(mcg_handle *h) {
   if (!h->checker_lds || h->fcc()) return false;
   plan_words_if_changed(h);
   return (!h->any_even() || h->even_words.oct) && (!h->any_ring() || h->ring_words.oct);
 }
+bool all_on_bits(mcg_handle const *h) {
+  if (h->checker_lds || h->fcc()) return false;
+  for (int c = 0; c < h->n_chains; ++c)
+    if (h->active[c] && !h->cring[c] && !bit_fits(h->cp[c])) return false;
+  return true;
+}
 
-// Autotuner cache key: path (LDS-resident or HBM), lattice, colouring and
-// the size class (log2 of the sites per chain and of the chain count).
-std::string tune_key(const mcg_handle *h) {
+// Autotuner cache key: path (words in LDS, bytes in LDS, bits or bytes in HBM: what suits
+// one says nothing of the others), lattice, colouring and the size class (log2 of the
+// sites per chain and of the chain count).
+std::string tune_key(mcg_handle *h) {
   int64_t sites = 0;
   for (int c = 0; c < h->n_chains; ++c) sites = std::max(sites, h->sites(c));
   auto lg = [](int64_t v) {
@@ -2141,7 +2149,11 @@ std::string tune_key(const mcg_handle *h) {
     while ((int64_t(1) << k) < v) ++k;
     return k;
   };
-  return std::string(h->checker_lds ? "lds" : "hbm") + ":" + std::to_string(h->lattice) + ":" +
+  const char *path = all_on_words(h)  ? "words"
+                     : h->checker_lds ? "lds"
+                     : all_on_bits(h) ? "bits"
+                                      : "hbm";
+  return std::string(path) + ":" + std::to_string(h->lattice) + ":" +
          std::to_string(h->ncolor) + ":" + std::to_string(lg(sites)) + ":" +
          std::to_string(lg(h->n_chains));
 }
