@@ -1792,26 +1792,34 @@ int rebuild_work(mcg_handle *h) {
   h->bit.n_items = 0;
   bool bit_ok = h->band_lines != 0 && !h->fcc();
   std::vector<BitItem> chains;
-  int64_t bit_total = 0;
+  int64_t bit_total = 0, bit_all = 0;
   h->bit_max_words = 0;
   for (int c = 0; c < h->n_chains && bit_ok; ++c) {
+    const int64_t words = h->cring[c] ? 0 : bit_words(h->cp[c]);
+    bit_all += std::max(words, h->capacity[c] / (h->lattice == MCG_LATTICE_SQUARE ? 16 : 32));
     if (!parity_chain(c)) continue;
     if (!bit_fits(h->cp[c])) bit_ok = false;
     chains.push_back({c, 0, 0, 0, bit_total});
-    const int64_t words = bit_words(h->cp[c]);
     h->bit_max_words = std::max(h->bit_max_words, words / (h->cp[c].ndim == 2 ? 2 : 1));
     bit_total += words;
   }
   if (bit_ok && bit_total > h->bit_cap) {
+    // at once for all the chains that the slots can hold, so that a larger active set
+    // does not free and allocate again: hipFree waits for everything on the device, other
+    // handles' runs too
     if (h->bit.bits) (void)hipFree(h->bit.bits);
     h->bit.bits = nullptr;
     h->bit_cap = 0;
-    if (hipMalloc(&h->bit.bits, sizeof(uint32_t) * (size_t)bit_total) == hipSuccess) {
-      h->bit_cap = bit_total;
-    } else {  // no room for the packed copies: the paths on the lattices themselves
+    for (const int64_t n : {std::max(bit_all, bit_total), bit_total}) {
+      if (hipMalloc(&h->bit.bits, sizeof(uint32_t) * (size_t)n) == hipSuccess) {
+        h->bit_cap = n;
+        break;
+      }
       (void)hipGetLastError();
-      bit_ok = false;
+      h->bit.bits = nullptr;
     }
+    // (no room for the packed copies: the paths on the lattices themselves)
+    if (h->bit_cap == 0) bit_ok = false;
   }
   if (bit_ok && bit_total > 0) {
     std::vector<BitItem> items;
