@@ -9,6 +9,8 @@
 // live in the caches -- and unpacks them at its end.
 #include "checker_bits.hh"
 
+#include <algorithm>
+
 namespace mcg {
 
 namespace {
@@ -911,22 +913,30 @@ int bit_plane_block(const CheckerParams &P, int oct) {
   return words >= 512 ? 512 : (words + 63) / 64 * 64;
 }
 
-static dim3 bit_copy_grid(int64_t max_words, int n_chains) {
-  return dim3((unsigned)((max_words + 255) / 256), (unsigned)n_chains);
+// (a grid's second dimension ends at 65535)
+template <typename Launch>
+static void bit_copy(int64_t max_words, int n_chains, Launch launch) {
+  for (int first = 0; first < n_chains; first += 65535)
+    launch(dim3((unsigned)((max_words + 255) / 256), (unsigned)std::min(65535, n_chains - first)),
+           first);
 }
 
 void launch_bit_pack(const CheckerParams *P, const CheckerState *St, const int8_t *lat_pool,
                      uint32_t *bits, const BitItem *chains, int n_chains, int64_t max_words,
                      hipStream_t stream) {
-  hipLaunchKernelGGL(bit_pack_kernel, bit_copy_grid(max_words, n_chains), dim3(256), 0, stream, P,
-                     St, lat_pool, bits, chains);
+  bit_copy(max_words, n_chains, [&](dim3 grid, int first) {
+    hipLaunchKernelGGL(bit_pack_kernel, grid, dim3(256), 0, stream, P, St, lat_pool, bits,
+                       chains + first);
+  });
 }
 
 void launch_bit_unpack(const CheckerParams *P, const CheckerState *St, int8_t *lat_pool,
                        const uint32_t *bits, const BitItem *chains, int n_chains,
                        int64_t max_words, hipStream_t stream) {
-  hipLaunchKernelGGL(bit_unpack_kernel, bit_copy_grid(max_words, n_chains), dim3(256), 0, stream,
-                     P, St, lat_pool, bits, chains);
+  bit_copy(max_words, n_chains, [&](dim3 grid, int first) {
+    hipLaunchKernelGGL(bit_unpack_kernel, grid, dim3(256), 0, stream, P, St, lat_pool, bits,
+                       chains + first);
+  });
 }
 
 int bit_pass_launches(const BitPass &b, BitLaunch (&L)[2]) {
