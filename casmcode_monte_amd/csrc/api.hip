@@ -1820,6 +1820,20 @@ int rebuild_work(mcg_handle *h) {
     h->bit_max_words = std::max(h->bit_max_words, words / (h->cp[c].ndim == 2 ? 2 : 1));
     bit_total += words;
   }
+  if (bit_ok && h->lattice == MCG_LATTICE_SC && h->ncolor == 8) {
+    // J1+J2: a workgroup updates a plane, a step of 512 words a colour, 19 us a pass for
+    // each step where the CUs have a plane or none; the line classes on bytes take 66 us
+    // and 4.5 more per 10^6 sites whatever the planes (MI355X, us a pass by planes and by
+    // classes: 512x512x2 84 and 68, 512x512x8 88 and 81, 640x512x16 105 and 91, 1024x340x40
+    // 113 and 118, 192x900x10 66 and 78)
+    int64_t sites = 0, steps = 0;
+    for (auto const &ch : chains) {
+      auto const &P = h->cp[ch.chain];
+      sites += P.n;
+      steps = std::max<int64_t>(steps, ((int64_t)(P.L1 / 2) * (P.L0 / 64) + 511) / 512);
+    }
+    if (sites < (steps - 3) * 4200000) bit_ok = false;
+  }
   if (bit_ok && bit_total > h->bit_cap) {
     // at once for all the chains that the slots can hold, so that a larger active set
     // does not free and allocate again: hipFree waits for everything on the device, other
