@@ -405,6 +405,7 @@ struct mcg_handle {
   // EXACT (and CANONICAL, which shares the state records d_xs)
   ExactParams *d_xp = nullptr;
   ExactState *d_xs = nullptr;
+  std::vector<ChainState> states;  // as last read (read_states)
   std::vector<ExactParams> xp;
   // per chain: LDS bytes of the block walk and whether they fit (else the
   // chain runs the scalar walk on its HBM lattice); device masks of the active
@@ -614,21 +615,18 @@ hipError_t copy_sync(mcg_handle *h, void *dst, const void *src, size_t n, hipMem
   return e != hipSuccess ? e : hipStreamSynchronize(h->stream);
 }
 
-// The sequential chains' states after a run, where the transfer puts them: in the staging
-// memory (until the next host copy), or in `own` if they do not fit it.  Copies of 64 KB
-// and more into memory of the call's own take the runtime two times, by what the process
-// copied before: 64 KMC chains, run_steps(1) 48 or 105 us, here 34; 256 chains 68 or 320,
-// here 46.
-hipError_t read_states(mcg_handle *h, std::vector<ExactState> &own, const ExactState *&xs) {
-  const size_t n = sizeof(ExactState) * (size_t)h->n_chains;
-  if (n <= 2 * STAGE_HALF) {
-    xs = reinterpret_cast<const ExactState *>(h->stage);
-    const hipError_t e = hipMemcpyAsync(h->stage, h->d_xs, n, hipMemcpyDeviceToHost, h->stream);
-    return e != hipSuccess ? e : hipStreamSynchronize(h->stream);
-  }
-  own.resize(h->n_chains);
-  xs = own.data();
-  return copy_sync(h, own.data(), h->d_xs, n, hipMemcpyDeviceToHost);
+// The sequential chains' states after a run, without their engines, which are nine tenths
+// of them.  Copies of all of it into memory of the call's own took the runtime one of two
+// times, by what the process had copied before: 64 KMC chains, run_steps(1) 48 or 105 us,
+// here 33; 256 chains 68 or 320, here 36; 2000 chains of 8x8, one pass 570 or 660, here 137.
+hipError_t read_states(mcg_handle *h) {
+  h->states.resize(h->n_chains);
+  return read_staged(h, h->states.data(), sizeof(ChainState) * h->states.size(),
+                     [&](int8_t *half, size_t first, size_t m) {
+                       launch_chain_states(h->d_xs, (int64_t)first / 8, (int64_t)m / 8,
+                                           reinterpret_cast<int64_t *>(half), h->stream);
+                       return hipGetLastError();
+                     });
 }
 
 hipError_t fill_sync(mcg_handle *h, void *dst, int v, size_t n) {
@@ -1319,9 +1317,8 @@ int kmc_run(mcg_handle *h, int64_t n_passes, int64_t n_steps,
   HIP_TRY(hipEventElapsedTime(&ms, h->ev0, h->ev1));
   h->last_ms = ms;
   h->last_attempts = events;
-  std::vector<ExactState> own;
-  const ExactState *xs = nullptr;
-  HIP_TRY(read_states(h, own, xs));
+  HIP_TRY(read_states(h));
+  auto const &xs = h->states;
   bool frozen = false;
   int64_t over = 0;
   h->kmc_pending = false;
@@ -2852,9 +2849,8 @@ int nfold_advance(mcg_handle *h, int64_t max_events, double stop_time, bool sele
   float ms = 0.f;
   HIP_TRY(hipEventElapsedTime(&ms, h->ev0, h->ev1));
   h->last_ms = ms;
-  std::vector<ExactState> own;
-  const ExactState *xs = nullptr;
-  HIP_TRY(read_states(h, own, xs));
+  HIP_TRY(read_states(h));
+  auto const &xs = h->states;
   bool frozen = false;
   double events = 0.0;
   for (int c = 0; c < h->n_chains; ++c) {
@@ -3003,9 +2999,8 @@ int occupant_run(mcg_handle *h, int64_t n_passes, int64_t n_steps) {
                               ? "Error in choose_canonical_swap: No events possible."
                               : "Error in choose_semigrand_canonical_swap: No events possible.";
   HIP_TRY(hipStreamSynchronize(h->stream));
-  std::vector<ExactState> own;
-  const ExactState *xs = nullptr;
-  HIP_TRY(read_states(h, own, xs));
+  HIP_TRY(read_states(h));
+  auto const &xs = h->states;
   int64_t need = 0;
   double attempts = 0.0;
   for (int c = 0; c < h->n_chains; ++c) {
@@ -3041,7 +3036,7 @@ int occupant_run(mcg_handle *h, int64_t n_passes, int64_t n_steps) {
   HIP_TRY(hipEventElapsedTime(&ms, h->ev0, h->ev1));
   h->last_ms = ms;
   h->last_attempts = attempts;
-  HIP_TRY(read_states(h, own, xs));
+  HIP_TRY(read_states(h));
   bool frozen = false;
   for (int c = 0; c < h->n_chains; ++c) {
     if (!h->active[c]) continue;
@@ -3205,9 +3200,8 @@ int mcg_run(mcg_handle *h, int64_t n_passes) {
     h->n_pass[c] = p0 + n_passes;
   }
   if (count_on_device) {
-    std::vector<ExactState> own;
-    const ExactState *xs = nullptr;
-    HIP_TRY(read_states(h, own, xs));
+    HIP_TRY(read_states(h));
+    auto const &xs = h->states;
     int64_t over = 0;
     for (int c = 0; c < h->n_chains; ++c) {
       if (!h->active[c]) continue;

@@ -1229,6 +1229,21 @@ void launch_checker_spins(const int8_t *lat, int64_t L0, int64_t first, int64_t 
                      first, count, out);
 }
 
+__global__ void chain_states_kernel(const ExactState *xs, int64_t first, int64_t count,
+                                    int64_t *out) {
+  constexpr int64_t WORDS = sizeof(ChainState) / 8;
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= count) return;
+  const ChainState *s = xs + (first + i) / WORDS;
+  out[i] = reinterpret_cast<const int64_t *>(s)[(first + i) % WORDS];
+}
+
+void launch_chain_states(const ExactState *xs, int64_t first, int64_t count, int64_t *out,
+                         hipStream_t stream) {
+  hipLaunchKernelGGL(chain_states_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0,
+                     stream, xs, first, count, out);
+}
+
 __global__ void clear_samples_kernel(ExactState *xs, CheckerState *cs, int n_chains) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= n_chains) return;

@@ -63,9 +63,12 @@ inline hipError_t set_dynamic_lds(const void *fn, int bytes, bool at_zero) {
   return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
 }
 
-// Read-write per-chain state (EXACT, CANONICAL and NFOLD).
-struct ExactState {
+// Read-write per-chain state of the sequential modes: the engine's words, and the rest,
+// which the host reads after a run (its bytes follow one another).
+struct EngineState {
   uint64_t mt[MT_N];  // std::mt19937_64 state words
+};
+struct ChainState {
   int64_t pos;        // index of the next output (312: twist first)
   int64_t n_pass, n_accept, n_reject;
   int64_t S, M;       // exact bond sum and magnetisation
@@ -94,6 +97,9 @@ struct ExactState {
   // time is in pending_dt
   int64_t kmc_pdir, kmc_pk;
 };
+struct ExactState : EngineState, ChainState {};
+static_assert(sizeof(ExactState) == sizeof(EngineState) + sizeof(ChainState) &&
+              sizeof(ChainState) % 8 == 0);
 
 // Every active chain makes n_passes * n + n_steps attempts from where it stands.
 void launch_exact(const ExactParams *P, ExactState *S, int8_t *lat_pool, mcg_sample *series,
@@ -396,6 +402,9 @@ void launch_checker_spins(const int8_t *lat, int64_t L0, int64_t first, int64_t 
 // Every chain's sample count to 0: of the sequential chains' states, or (xs null) of
 // the checkerboard ones'.
 void launch_clear_samples(ExactState *xs, CheckerState *cs, int n_chains, hipStream_t stream);
+// Words [first, first + count) of the chains' ChainStates, one after another, into out.
+void launch_chain_states(const ExactState *xs, int64_t first, int64_t count, int64_t *out,
+                         hipStream_t stream);
 
 // the state, counter and records of the last `passes` passes (at most CHECKER_AHEAD)
 void launch_checker_record(CheckerState *St, int64_t *parts, mcg_sample *series,

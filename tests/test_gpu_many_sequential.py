@@ -1,6 +1,6 @@
-"""Handles of so many sequential chains that the read-back of their states takes one way or
-another (64 KB, and the 1 MB of staging memory, lie between): positions, records and
-counters of every chain follow runs that differ from chain to chain."""
+"""Handles of one to so many sequential chains that the read-back of their states goes through
+the staging memory in parts: positions, records and counters of every chain follow runs that
+differ from chain to chain."""
 import numpy as np
 import pytest
 
@@ -9,7 +9,7 @@ import casmcode_monte_amd as M
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("chains", [1, 24, 25, 390, 400])
+@pytest.mark.parametrize("chains", [1, 24, 25, 390, 400, 2600, 5200])
 @pytest.mark.parametrize("mode", ["kmc", "occupant", "nfold"])
 def test_states_of_every_chain(mode, chains):
     print("many sequential", mode, chains, flush=True)
