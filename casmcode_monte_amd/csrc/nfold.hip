@@ -444,7 +444,10 @@ __global__ __launch_bounds__(64) void nfold_kernel(const NfoldParams *__restrict
     dS += -s_old * (nsum - self_nb * s_old) / 2;
     dM -= s_old;
     // the flip itself is written with l's move (its spin bit follows its class)
-#pragma unroll 1
+    // (only narrow lattices take these moves event after event: 1x3000, two passes 10.0 ms
+    // in a loop and 7.5 unrolled)
+    constexpr int UNROLL = GENERAL ? 5 : 1;
+#pragma unroll UNROLL
     for (int t = 0; t < 5; ++t) {
       const uint32_t x = (uint32_t)__builtin_amdgcn_readlane((int)xs, t);
       const int a = __builtin_amdgcn_readlane(c_pre, t), b = __builtin_amdgcn_readlane(c_post, t);
