@@ -394,7 +394,6 @@ def bench_checker_scan(passes):
     conds = c2_conditions()
     b = cm.Run(conds, mode=cm.MODE_CHECKERBOARD, J1=0.1, J2=0.0)
     b.run(5)
-    sched = b.autotune(20)
     bw, bk, ba = timed_run(b, passes)
     b.close()
     plain_wall, plain_att = 0.0, 0.0
@@ -407,7 +406,6 @@ def bench_checker_scan(passes):
         p.close()
     lds_gbs = 6.0 * ba / bk / 1e9  # own read + 4 neighbour reads + write per attempt
     return dict(passes=passes, batched_attempts_per_s=ba / bw, batched_kernel_s=bk,
-                lds_block=sched["lds_block"],
                 plain_attempts_per_s=plain_att / plain_wall,
                 ratio=(ba / bw) / (plain_att / plain_wall),
                 roofline={"bound": "lds", "achieved": lds_gbs, "peak": LDS_PEAK["gbs"],
