@@ -574,9 +574,9 @@ __global__ __launch_bounds__(CUBE_BLOCK) void checker_cube_kernel(
 // the record while the others go on.
 //
 // Measured on MI355X, us a pass, against the workgroups on bytes (checker_lds_kernel,
-// checker_ring_lds_kernel): 64 chains of 128x128 2.8 and 6.6, one of 32x32 1.7 and 3.8,
-// 64 of 250x250 6.6 and 101 (lines that are no multiple of 32 took 4 sites a thread
-// and byte loads), 64 of 181x253 18 and 64, 64 of 31x45 10 and 12.  A step of the
+// checker_ring_lds_kernel): 64 chains of 128x128 2.6 and 6.6, one of 32x32 1.5 and 3.8,
+// 64 of 250x250 6.4 and 101 (lines that are no multiple of 32 took 4 sites a thread
+// and byte loads), 64 of 181x253 12 and 64, 64 of 31x45 6 and 12.  A step of the
 // smallest is the latency of one word's chain and a barrier, ~1 us.
 // ---------------------------------------------------------------------------
 template <bool RING, bool NNN, int OCT>

@@ -1,5 +1,5 @@
 // exact.hip -- EXACT mode: the reference's sequential random-site Metropolis
-// chain, reproduced bit for bit on one wavefront per chain.
+// chain, reproduced bit for bit by one walking wavefront per chain.
 //
 // Reference: the main loop of basic_occupation_metropolis.hh:381-422 driving the
 // SGC Ising calculator (basic_semigrand_canonical.hh:308-320 propose/apply,

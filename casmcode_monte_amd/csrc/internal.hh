@@ -12,7 +12,7 @@
 namespace mcg {
 
 // ---------------------------------------------------------------------------
-// EXACT mode: one chain per 64-lane workgroup (one wavefront).
+// EXACT mode: a chain per workgroup, of one wave (scalar walk) or five (block walk).
 // ---------------------------------------------------------------------------
 
 // Number of (old spin, neighbour sum) classes of the 2D square NN Ising flip:
@@ -110,7 +110,7 @@ void launch_exact(const ExactParams *P, ExactState *S, int8_t *lat_pool, mcg_sam
 // ---------------------------------------------------------------------------
 // OCCUPANT mode: occupant events over an OccLocation with several asymmetric
 // units (semi-grand canonical single-site events or canonical pair swaps),
-// one chain per wavefront.
+// a chain per workgroup of two (general kernel) or five waves.
 // ---------------------------------------------------------------------------
 constexpr int OCC_MAX_ASYM = 8;
 constexpr int OCC_MAX_CAND = 2 * OCC_MAX_ASYM;
@@ -167,7 +167,7 @@ hipError_t occupant_set_max_lds(int general_bytes, int sgc_bytes);
 
 // ---------------------------------------------------------------------------
 // KMC mode: kinetic Monte Carlo with atom tracking for a square lattice gas,
-// one chain per wavefront.
+// a chain per workgroup of two (general kernel) or five waves.
 // ---------------------------------------------------------------------------
 // classes of a hop: a - b + 3 (a, b: atoms next to the origin other than at
 // the target, next to the target other than at the origin), dE = J (a - b)
@@ -229,7 +229,7 @@ void launch_kmc(const KmcParams *P, ExactState *S, int8_t *lat_pool, int32_t *li
 hipError_t kmc_set_max_lds(int general_bytes, int walk_bytes);
 
 // ---------------------------------------------------------------------------
-// CANONICAL mode: pair swaps at fixed composition, one chain per wavefront.
+// CANONICAL mode: pair swaps at fixed composition, a chain per workgroup of five waves.
 // ---------------------------------------------------------------------------
 
 // Classes of a swap (site a: -1 -> +1, then site b: +1 -> -1): the neighbour

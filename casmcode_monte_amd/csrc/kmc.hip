@@ -1,8 +1,8 @@
 // kmc.hip -- KMC mode: kinetic Monte Carlo with atom tracking for a square
 // lattice gas, bit for bit the loop of kinetic_monte_carlo.hh:136-229 under a
-// rejection event selector, on one wavefront per chain; a second wavefront of
-// the workgroup twists the engine's next generation meanwhile (mt_producer,
-// walk.hh).
+// rejection event selector, by one walking wavefront per chain.  In kmc_kernel a
+// second one twists the engine's next generation meanwhile (mt_producer, walk.hh);
+// kmc_walk_kernel has four more waves.
 //
 // Model: occupant 0 = vacancy, 1 = atom, E = -J sum over nearest-neighbour
 // bonds of n_i n_j.  Selector: attempts follow one another at 1/R, R = 4 *

@@ -1,8 +1,9 @@
 // occupant.hip -- OCCUPANT mode: the reference's generic occupant-event
 // Metropolis chain over an OccLocation with several asymmetric units, for
 // semi-grand canonical single-site events or canonical pair swaps, reproduced
-// bit for bit on one wavefront per chain; a second wavefront of the workgroup
-// twists the engine's next generation meanwhile (mt_producer, walk.hh).
+// bit for bit by one walking wavefront per chain.  In occupant_kernel a second one
+// twists the engine's next generation meanwhile (mt_producer, walk.hh);
+// occupant_sgc_kernel has four more waves.
 //
 // Reference: the loop of occupation_metropolis.hh:87-153 with
 // propose_semigrand_canonical_event (OccEventProposal.hh:261-352) or
@@ -516,7 +517,7 @@ __global__ __launch_bounds__(128) void occupant_kernel(
 // split and with it half of the later steps' slots.
 //
 // Measured on MI355X, 64 chains of 128x128 sites over two units, 131072 steps each:
-// 74.7 ms by occupant_kernel, 24.0 ms here (1370 and 450 cycles a step at 2.4 GHz
+// 74.7 ms by occupant_kernel, 23.5 ms here (1370 and 450 cycles a step at 2.4 GHz
 // for the chain that accepts most, 45 for the coldest): a block per accepted step,
 // its time the chain record -> list entry -> class byte -> starts -> next record.
 // The starts come from one scan of the window, not an attempt at a time: 28.1 ms and

@@ -1,8 +1,9 @@
 // walk.hh -- wavefront helpers shared by the sequential-chain kernels (EXACT
-// single-site flips, canonical pair swaps, N-fold way): scalar broadcasts, the
-// out-of-place MT19937-64 twist into a ring of tempered outputs, and the
-// producer/consumer hand-off through which a second wavefront twists the
-// engine while the walking wavefront consumes it.
+// single-site flips, canonical pair swaps, occupant events, KMC, N-fold way): scalar
+// broadcasts, the out-of-place MT19937-64 twist, and the hand-offs by which other
+// waves of the workgroup work beside the walking one: one that twists the engine into
+// a ring of tempered outputs (the general OCCUPANT and KMC kernels), or three that
+// twist it and leave a record per word, and one that adds energies and writes samples.
 #pragma once
 
 #include <hip/hip_runtime.h>
