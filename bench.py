@@ -622,9 +622,9 @@ def main():
         "data": "synthetic (all +1 initial lattices, seeded MT19937-64 streams)",
         "config": {"workload": "batched exact mode: 2D Ising 128x128, J=0.1 eV, 64 chains "
                                "(8 T in 500-3000 K x 8 mu in -0.4..0.4 eV), seeds 1000+i, "
-                               "MT19937-64, FP64 running energy, one chain per wavefront",
+                               "MT19937-64, FP64 running energy, one chain per workgroup",
                    "chains": 64, "sites_per_chain": 16384, "passes": K,
-                   "parallelism": "1 GPU, 64 workgroups (one 64-lane wavefront per chain)"},
+                   "parallelism": "1 GPU, 64 workgroups (a chain each, walked by one of five wavefronts)"},
         "roofline": {"bound": "latency", "achieved": lds_achieved, "peak": LDS_PEAK["gbs"],
                      "unit": "GB/s", "frac": lds_achieved / LDS_PEAK["gbs"],
                      "peak_source": LDS_PEAK["source"],

@@ -463,7 +463,7 @@ struct mcg_handle {
   bool kmc_pending = false;  // a chain may hold a pending event
   int64_t kmc_spin_limit = int64_t(1) << 26;
   bool kmc() const { return mode == MCG_MODE_KMC; }
-  // one sequential chain per wavefront, MT19937-64 state, native lattice layout
+  // one sequential chain per workgroup, MT19937-64 state, native lattice layout
   bool sequential() const {
     return mode == MCG_MODE_EXACT || mode == MCG_MODE_CANONICAL || mode == MCG_MODE_NFOLD ||
            mode == MCG_MODE_OCCUPANT || mode == MCG_MODE_KMC;

@@ -35,14 +35,14 @@ extern "C" {
 #define MCG_ERR_CAPACITY 4 /* caller buffer too small / device memory exhausted */
 
 /* ---- modes and lattices ----------------------------------------------------- */
-/* EXACT: one sequential chain per wavefront that reproduces the reference's
+/* EXACT: one sequential chain per workgroup that reproduces the reference's
  *   random-site order and std::mt19937_64 stream bit for bit
  *   (basic_occupation_metropolis.hh:381-422 with the event generator of
  *   basic_semigrand_canonical.hh:308-320).  Square lattice, J1 only.
  * CHECKERBOARD: sublattice-coloured sweeps with a Philox4x32-10 counter RNG;
  *   one pass updates every site once.  Square (2D) or simple-cubic (3D)
  *   lattices with nearest (J1) and next-nearest (J2) couplings.
- * CANONICAL: one sequential chain per wavefront running the reference's
+ * CANONICAL: one sequential chain per workgroup running the reference's
  *   canonical pair-swap Metropolis bit for bit: the generic loop of
  *   occupation_metropolis.hh:87-153 with propose_canonical_event
  *   (OccEventProposal.hh:109-236) over an OccLocation (OccLocation.cc:39-118,
@@ -73,7 +73,7 @@ extern "C" {
  *   On the time grid, a chain whose total rate reaches 0 (every flip's
  *   probability underflows) fails the run with MCG_ERR_STATE. */
 #define MCG_MODE_NFOLD 3
-/* OCCUPANT: one sequential chain per wavefront running the reference's generic
+/* OCCUPANT: one sequential chain per workgroup running the reference's generic
  *   occupant-event Metropolis bit for bit: the loop of
  *   occupation_metropolis.hh:87-153 over an OccLocation (OccLocation.cc:39-118,
  *   216-283) with several asymmetric units, proposing either semi-grand
@@ -509,7 +509,7 @@ int mcg_check_batch(mcg_handle *h, int64_t n, const int64_t *chains, int64_t obs
                     double prec, double confidence, mcg_check *out);
 
 /* Launch schedule of a CHECKERBOARD handle (EXACT handles have nothing to
- * tune: one wavefront per chain).  Every schedule produces the same
+ * tune: a walking wavefront per chain).  Every schedule produces the same
  * trajectories; only the speed changes. */
 typedef struct mcg_schedule {
   int64_t lds_block;        /* FCC and LDS-resident kernels on bytes: threads per workgroup
